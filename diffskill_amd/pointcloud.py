@@ -223,8 +223,9 @@ def epsilon_schedule(x, y, p, blur, scaling):
 
 
 def _sinkhorn_work(x, y):
-    """Scratch of one call on the current stream (the allocator hands its memory
-    on in that stream's order)."""
+    """Scratch of one call on the current stream.  The caller holds it until the
+    call has returned: its launches are issued without the GIL, and a tensor let
+    go before them could be handed to another thread's launches in between."""
     nb = _lib.load().pc_sinkhorn_step_work_bytes(x.shape[0], y.shape[0])
     return torch.empty((nb + 15) // 16 * 4, dtype=torch.float32, device=x.device)
 
@@ -240,8 +241,9 @@ class _SinkhornDivergence(torch.autograd.Function):
         pot = torch.empty(4 * (N + M), dtype=torch.float32, device=xd.device)
         loss = torch.empty((), dtype=torch.float32, device=xd.device)
         eps = (ctypes.c_float * len(eps_s))(*eps_s)
+        work = _sinkhorn_work(xd, yd)
         _check("pc_sinkhorn_solve", _lib.load().pc_sinkhorn_solve(_p(xd), N, _p(yd), M, eps, len(eps_s), p, _p(pot), _p(loss),
-                                                                  _p(_sinkhorn_work(xd, yd)), _stream()))
+                                                                  _p(work), _stream()))
         ctx.clouds, ctx.pot, ctx.eps, ctx.p = (xd, yd), pot, eps_s[-1], p
         return loss.to(x.dtype)
 
@@ -253,9 +255,10 @@ class _SinkhornDivergence(torch.autograd.Function):
         # a gradient that is to be differentiated again (in go) takes the factor
         # outside the kernel
         inside = go.detach().to(torch.float32) if not go.requires_grad else None
+        work = _sinkhorn_work(xd, yd)
         _check("pc_sinkhorn_grad", _lib.load().pc_sinkhorn_grad(
             _p(xd), xd.shape[0], _p(yd), yd.shape[0], _p(ctx.pot), ctx.eps, ctx.p, None if inside is None else _p(inside),
-            *(None if g is None else _p(g) for g in (gx, gy)), _p(_sinkhorn_work(xd, yd)), _stream()))
+            *(None if g is None else _p(g) for g in (gx, gy)), _p(work), _stream()))
         if inside is None:
             gx, gy = (None if g is None else g * go for g in (gx, gy))
         return (*(None if g is None else g.to(go.dtype) for g in (gx, gy)), None, None, None)
