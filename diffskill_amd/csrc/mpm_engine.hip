@@ -931,14 +931,26 @@ DEV void scatter_tile(float4* tile, float* stage, const ScatLane& sl, ScatAcc& a
     if (act == 0ull) return;
     float* sp = stage + (lane & 3) * 16 + (lane >> 2);
     f4 w0[4], w1[4], bq[4];
+    // A lane that takes no part may be anywhere, at infinity too, and one that
+    // does may be at NaN (binned into cell 0): their weights count as 0, which
+    // the zeroed columns then keep out of the other cells of their 16 lanes.
+    // NaN columns (u's are, by its own formula) carry it into its own cell.
+    float ws = sw.w[0][0] + sw.w[0][1] + sw.w[0][2];
+    bool num = valid && ws == ws;
+    float w[3][3];
+#pragma unroll
+    for (int o = 0; o < 3; o++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) w[o][d] = num ? sw.w[o][d] : 0.f;
+    if (NCOMP == 4 && !num) mass = ws;
     // (LDS operations of one wave complete in order; the fences keep the
     // compiler from moving reads and writes of the stage across each other)
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 #pragma unroll
     for (int a = 0; a < 3; a++) {
 #pragma unroll
-        for (int b = 0; b < 3; b++) sp[(a * 3 + b) * ST_ROW] = sw.w[a][0] * sw.w[b][1];
-        sp[(9 + a) * ST_ROW] = sw.w[a][2];
+        for (int b = 0; b < 3; b++) sp[(a * 3 + b) * ST_ROW] = w[a][0] * w[b][1];
+        sp[(9 + a) * ST_ROW] = w[a][2];
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 #pragma unroll
