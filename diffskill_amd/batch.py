@@ -12,7 +12,7 @@ import numpy as np
 import torch
 
 from .config import derive
-from .engine.core import Engine, cell_sort_perm, l1_rows, scene_desc
+from .engine.core import Engine, cell_sort_perm, l1_rows, l1_rows_takes, scene_desc
 from .engine.mpm_simulator import collision_pairs, collision_rand
 from .engine.primitive.primitives import CLASSES
 
@@ -224,7 +224,7 @@ class BatchedTrajOpt:
 
     def losses(self):
         m, t = self.mass, self.targets
-        if m.shape == t.shape and m.dtype == t.dtype == torch.float32 and m.device == t.device and not t.requires_grad:
+        if l1_rows_takes(m, t) and not t.requires_grad:
             return l1_rows(m, t)
         return (m - t).abs().sum(dim=(1, 2, 3))
 

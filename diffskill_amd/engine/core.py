@@ -55,9 +55,17 @@ def pack_state(x, v, C, F, perm, stride, col):
     return soa
 
 
+def l1_rows_takes(a, b):
+    """Whether l1_rows takes these two: it reads both as one run of values a row."""
+    return (isinstance(b, torch.Tensor) and a.is_cuda and a.device == b.device and a.shape == b.shape and a.dtype == b.dtype == torch.float32
+            and a.is_contiguous() and b.is_contiguous() and a.dim() > 0 and len(a) <= 65535)
+
+
 def l1_rows(a, b):
     """(a - b).abs().sum over all dimensions but the first, float32, of two
     contiguous float32 device tensors of one shape; summed in 64 bits."""
+    if not l1_rows_takes(a, b):
+        raise ValueError("l1_rows takes contiguous float32 device tensors of one shape and at most 65535 rows")
     rows = a.shape[0]
     work = torch.empty((max(1, rows), 256), dtype=torch.float64, device=a.device)
     out = torch.empty(rows, dtype=torch.float32, device=a.device)
