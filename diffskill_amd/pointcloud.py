@@ -211,8 +211,8 @@ def epsilon_schedule(x, y, p, blur, scaling):
     exp(arange(p log d, p log blur, p log scaling)), then blur^p.  A diagonal
     below blur (all points within blur of each other) is taken as blur, so the
     schedule is just blur^p twice instead of starting at eps = 0."""
-    if (x.is_cuda and x.device == y.device and x.dtype == y.dtype == torch.float32 and x.is_contiguous()
-            and y.is_contiguous()):
+    if (x.is_cuda and x.device == y.device and x.dtype == y.dtype == torch.float32 and x.is_contiguous() and y.is_contiguous()
+            and x.dim() == y.dim() == 2 and x.shape[1] == y.shape[1] == 3):   # (rows of three are what the kernel reads)
         ext = torch.empty(3, dtype=torch.float32, device=x.device)
         _check("pc_extent", _lib.load().pc_extent(_p(x), x.shape[0], _p(y), y.shape[0], _p(ext), _stream()))
     else:
