@@ -27,10 +27,25 @@ def cell_sort_perm(x, n_grid):
 
 
 def cell_order(x, n_grid, out=None):
-    """cell_sort_perm and its inverse, (2, n) int64 (into ``out`` when given)."""
-    x = np.ascontiguousarray(np.asarray(x, np.float64).reshape(-1, 3))
+    """cell_sort_perm and its inverse, (2, n) int64 (into ``out`` when given),
+    of rows whose first three columns are positions."""
+    x = np.asarray(x, np.float64)
+    if x.ndim == 1 and x.size == 0:   # (an empty list)
+        x = x.reshape(0, 3)
+    if x.ndim != 2 or x.shape[1] < 3:
+        raise ValueError("positions must be (n, 3), got %s" % (x.shape,))
+    x = np.ascontiguousarray(x[:, :3])
     if out is None:
         out = np.empty((2, len(x)), np.int64)
+    if out.shape != (2, len(x)) or out.dtype != np.int64 or not out.flags.c_contiguous:
+        raise ValueError("out must be a contiguous (2, %d) int64 array" % len(x))
+    if n_grid > 2048:   # (more cells than mpm_cell_order's keys hold)
+        b = np.clip(np.trunc(x * n_grid - 0.5).astype(np.int64), 0, n_grid - 1)
+        nb = (n_grid + 3) // 4
+        blk = ((b[:, 0] >> 2) * nb + (b[:, 1] >> 2)) * nb + (b[:, 2] >> 2)
+        out[0] = np.argsort(blk * 64 + ((b[:, 0] & 3) << 4 | (b[:, 1] & 3) << 2 | (b[:, 2] & 3)), kind="stable")
+        out[1, out[0]] = np.arange(len(x))
+        return out
     _lib.check(_lib.load().mpm_cell_order(ctypes.c_void_p(x.ctypes.data), len(x), int(n_grid), ctypes.c_void_p(out[0].ctypes.data),
                                           ctypes.c_void_p(out[1].ctypes.data)), "mpm_cell_order")
     return out
