@@ -2791,6 +2791,7 @@ struct mpm_ctx {
     long long n_nodes = 0, n_particles = 0;
     std::vector<SceneC> scenes;
     std::vector<PrimC> prims;
+    bool prims_uploaded = true;   // the device holds `prims` (mpm_create returns no context otherwise)
     std::vector<int> p_off;
     SceneC* d_scenes = nullptr;
     PrimC* d_prims = nullptr;
@@ -4087,17 +4088,22 @@ int mpm_pack_state(const float* x, const float* v, const float* C, const float* 
 
 int mpm_update_prims(mpm_ctx* ctx, const mpm_prim_desc* prims, void* stream) {
     if (!ctx || (!prims && ctx->n_prims > 0)) return fail("mpm_update_prims: null argument");
-    bool same = true;
-    for (int q = 0; q < ctx->n_prims; q++) {
+    for (int q = 0; q < ctx->n_prims; q++)
         if (prims[q].type != ctx->prims[q].type) return fail("mpm_update_prims: primitive types may not change");
+    // unchanged constants that the device is known to hold are not uploaded again;
+    // until an upload has gone through, ctx->prims says nothing about the device
+    bool same = ctx->prims_uploaded;
+    for (int q = 0; q < ctx->n_prims; q++) {
         PrimC p = to_primc(prims[q]);
         same = same && std::memcmp(&p, &ctx->prims[q], sizeof(PrimC)) == 0;
-        ctx->prims[q] = p;
     }
     ctx->drop_kept();  // kept grids were built with the old primitive parameters
-    if (ctx->n_prims == 0 || same) return 0;   // (unchanged: the device has them)
+    if (ctx->n_prims == 0 || same) return 0;
+    ctx->prims_uploaded = false;
+    for (int q = 0; q < ctx->n_prims; q++) ctx->prims[q] = to_primc(prims[q]);
     HIPCHK(hipMemcpyAsync(ctx->d_prims, ctx->prims.data(), sizeof(PrimC) * ctx->n_prims, hipMemcpyHostToDevice, S_(stream)));
     HIPCHK(hipStreamSynchronize(S_(stream)));
+    ctx->prims_uploaded = true;
     return 0;
 }
 
