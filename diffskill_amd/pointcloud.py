@@ -241,7 +241,6 @@ class _SinkhornDivergence(torch.autograd.Function):
         pot = torch.empty(4 * (N + M), dtype=torch.float32, device=xd.device)
         loss = torch.empty((), dtype=torch.float32, device=xd.device)
         eps = (ctypes.c_float * len(eps_s))(*eps_s)
-        p = int(p)   # (2.0 and numpy's integers too)
         work = _sinkhorn_work(xd, yd)
         _check("pc_sinkhorn_solve", _lib.load().pc_sinkhorn_solve(_p(xd), N, _p(yd), M, eps, len(eps_s), p, _p(pot), _p(loss),
                                                                   _p(work), _stream()))
