@@ -50,6 +50,15 @@ def _p(t):
     return ctypes.c_void_p(t.data_ptr())
 
 
+def _has_memory(t):
+    """Whether a kernel can read t: a gradient batched by vmap has no memory of its own."""
+    try:
+        t.data_ptr()
+        return True
+    except RuntimeError:
+        return False
+
+
 def _check(name, rc):
     if rc != 0:
         raise RuntimeError("%s failed: %s" % (name, _lib.load().pc_last_error().decode(errors="replace")))
@@ -94,7 +103,7 @@ def _distance_grad(x, y, idx, d, squared, g, want_y):
     else:
         inv = torch.where(d > 0, 1.0 / d.clamp_min(1e-30), torch.zeros_like(d))
         gx = diff * (g * inv.to(g.dtype))[:, None]
-    return gx, torch.zeros_like(y).index_add_(0, idx, -gx) if want_y else None
+    return gx, torch.zeros_like(y).index_add(0, idx, -gx) if want_y else None
 
 
 class _NearestDistance(torch.autograd.Function):
@@ -157,8 +166,9 @@ class _Chamfer(torch.autograd.Function):
         x, y, ix, dx, iy, dy = ctx.saved_tensors
         want = ctx.needs_input_grad
         n, m = x.shape[0], y.shape[0]
-        if torch.is_grad_enabled():
-            # a gradient that is to be differentiated again: in operations that are
+        if torch.is_grad_enabled() or not _has_memory(go):
+            # a gradient that is to be differentiated again, or a batch of them: in
+            # operations that take those
             def one(p, t, idx, d2, w):
                 return _distance_grad(p, t, idx.long(), d2 if ctx.squared else torch.sqrt(d2), ctx.squared,
                                       (go / p.shape[0]).expand(p.shape[0]), w)
@@ -252,9 +262,9 @@ class _SinkhornDivergence(torch.autograd.Function):
         xd, yd = ctx.clouds
         want = ctx.needs_input_grad[:2]
         gx, gy = (torch.empty_like(c) if w else None for c, w in zip((xd, yd), want))
-        # a gradient that is to be differentiated again (in go) takes the factor
-        # outside the kernel
-        inside = go.detach().to(torch.float32) if not go.requires_grad else None
+        # a gradient that is to be differentiated again (in go), or a batch of them,
+        # takes the factor outside the kernel
+        inside = go.to(torch.float32) if not go.requires_grad and _has_memory(go) else None
         work = _sinkhorn_work(xd, yd)
         _check("pc_sinkhorn_grad", _lib.load().pc_sinkhorn_grad(
             _p(xd), xd.shape[0], _p(yd), yd.shape[0], _p(ctx.pot), ctx.eps, ctx.p, None if inside is None else _p(inside),

@@ -1,5 +1,6 @@
 """The host side of the point-cloud losses, with the library's entry points
 replaced by stand-ins that look at what they are given."""
+import ctypes
 import weakref
 
 import pytest
@@ -53,3 +54,51 @@ def test_sinkhorn_scratch_lives_through_the_call(host, monkeypatch):
     x, y = torch.rand(5, 3, requires_grad=True), torch.rand(4, 3)
     pc.sinkhorn_divergence(x, y).backward()
     assert alive == [True, True]
+
+
+def _zeros(p, nbytes):
+    if p is not None:
+        ctypes.memset(p, 0, nbytes)
+    return 0
+
+
+def _search(x, n, y, m, work, ix, dx, iy, dy, stream):
+    """Every point's nearest target is target 0, at distance 0."""
+    return _zeros(ix, 4 * n) or _zeros(dx, 4 * n) or _zeros(iy, 4 * m) or _zeros(dy, 4 * m)
+
+
+def _chamfer_library():
+    return Library(pc_nearest_pair_work_bytes=64, pc_nearest_pair=_search)
+
+
+@pytest.mark.parametrize("both", [False, True])
+def test_chamfer_batch_of_gradients(host, both):
+    """Several gradients of one loss at once (vmap over the backward)."""
+    lib = host(_chamfer_library())
+    x, y = torch.rand(5, 3, requires_grad=True), torch.rand(4, 3, requires_grad=True)
+    loss = pc.chamfer_distance(x, y, bidirectional=both)
+    gx, gy = torch.autograd.grad(loss, (x, y), torch.tensor([1.0, -2.0]), is_grads_batched=True)
+    ref = 2 * (x - y[0]) / 5
+    add = torch.zeros(4, 3).index_add(0, torch.zeros(5, dtype=torch.long), -ref)
+    if both:
+        hy = 2 * (y - x[0]) / 4
+        ref, add = ref.index_add(0, torch.zeros(4, dtype=torch.long), -hy), add + hy
+    for k, f in enumerate((1.0, -2.0)):
+        assert torch.allclose(gx[k], f * ref) and torch.allclose(gy[k], f * add)
+
+
+def test_sinkhorn_batch_of_gradients(host):
+    def grad(x, n, y, m, pot, eps, p, go, gx, gy, work, stream):
+        f = 1.0 if go is None else ctypes.cast(go, ctypes.POINTER(ctypes.c_float))[0]
+        for g, k in ((gx, n), (gy, m)):
+            if g is not None:
+                ctypes.memmove(g, (ctypes.c_float * (3 * k))(*([f] * (3 * k))), 12 * k)
+        return 0
+
+    host(Library(pc_sinkhorn_step_work_bytes=4096, pc_sinkhorn_grad=grad))
+    x, y = torch.rand(5, 3, requires_grad=True), torch.rand(4, 3, requires_grad=True)
+    loss = pc.sinkhorn_divergence(x, y)
+    one = torch.autograd.grad(loss, (x, y), torch.tensor(0.5), retain_graph=True)
+    got = torch.autograd.grad(loss, (x, y), torch.tensor([1.0, -2.0]), is_grads_batched=True)
+    for a, b in zip(one, got):
+        assert (a == 0.5).all() and (b[0] == 1.0).all() and (b[1] == -2.0).all()
