@@ -166,9 +166,10 @@ class _Chamfer(torch.autograd.Function):
         x, y, ix, dx, iy, dy = ctx.saved_tensors
         want = ctx.needs_input_grad
         n, m = x.shape[0], y.shape[0]
-        if torch.is_grad_enabled() or not _has_memory(go):
-            # a gradient that is to be differentiated again, or a batch of them: in
-            # operations that take those
+        if torch.is_grad_enabled() or not _has_memory(go) or torch.are_deterministic_algorithms_enabled():
+            # a gradient that is to be differentiated again, a batch of them, or one
+            # summed in a fixed order (pc_chamfer_grad's sums over the points that
+            # share a target have none): in operations that take those
             def one(p, t, idx, d2, w):
                 return _distance_grad(p, t, idx.long(), d2 if ctx.squared else torch.sqrt(d2), ctx.squared,
                                       (go / p.shape[0]).expand(p.shape[0]), w)

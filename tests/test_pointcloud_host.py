@@ -102,3 +102,18 @@ def test_sinkhorn_batch_of_gradients(host):
     got = torch.autograd.grad(loss, (x, y), torch.tensor([1.0, -2.0]), is_grads_batched=True)
     for a, b in zip(one, got):
         assert (a == 0.5).all() and (b[0] == 1.0).all() and (b[1] == -2.0).all()
+
+
+@pytest.mark.parametrize("fixed", [False, True])
+def test_chamfer_gradient_of_deterministic_algorithms(host, fixed):
+    """The gradient kernel's sums have no fixed order: not where one is asked for."""
+    lib = host(_chamfer_library())
+    x, y = torch.rand(5, 3, requires_grad=True), torch.rand(4, 3, requires_grad=True)
+    torch.use_deterministic_algorithms(fixed)
+    try:
+        gx, gy = torch.autograd.grad(pc.chamfer_distance(x, y), (x, y))
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert ("pc_chamfer_grad" in lib.seen) != fixed
+    if fixed:
+        assert torch.allclose(gx, 2 * (x - y[0]) / 5) and torch.allclose(gy[0], -gx.sum(0)) and (gy[1:] == 0).all()
