@@ -460,8 +460,9 @@ class Primitives:
         t = self._step_actions.get(s)
         if t is None:
             t = np.zeros((max(1, self.n), 7), np.float32)
-        elif isinstance(t, torch.Tensor):
-            t = t.cpu().numpy()
+        elif isinstance(t, tuple):   # (a device table and the stream that fills it)
+            torch.cuda.current_stream().wait_stream(t[1])
+            t = t[0].cpu().numpy()
         self._step_actions[s] = t
         return t
 
@@ -487,7 +488,7 @@ class Primitives:
                 lo, hi = self.action_dims[i:i + 2]
                 if hi > lo:
                     t[i, :hi - lo] = a[lo:hi]
-            self._step_actions[s] = t
+            self._step_actions[s] = (t, torch.cuda.current_stream())
             self._sim._set_actions(s, n_substeps, t)
             return
         if isinstance(action, torch.Tensor):
