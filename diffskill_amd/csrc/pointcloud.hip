@@ -85,8 +85,10 @@ __global__ void __launch_bounds__(PC_WG) k_pc_nearest(const float* __restrict__ 
 
 // ------------------------------------------------- nearest, spatially sorted
 // The same results with most pairs left out.  Both clouds are sorted along a
-// Morton curve of 16^3 cells over their own bounding box (counting sort), cut
-// into blocks of 32 points with their bounding boxes, and a workgroup finds the
+// Morton curve of 16^3 cells over their own extent (counting sort; a few points far
+// outside the others do not count for the extent and share its border cells, those
+// with a NaN or infinite coordinate count nowhere), cut into blocks of 32 points
+// with their bounding boxes, and a workgroup finds the
 // targets of a block of queries: the target block nearest to it and its
 // neighbours give every query an upper bound, blocks whose box is further from
 // the queries' box than the largest bound are dropped, then those that no
@@ -118,6 +120,8 @@ struct NnCloud {
 };
 struct NnPair { NnCloud c[2]; };
 
+// (no target is at a finite distance from it, and no query has it as its nearest)
+DEV_PC bool nn_special(float x, float y, float z) { return !(fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY); }
 DEV_PC int nn_spread(int v) { return (v & 1) | (v & 2) << 2 | (v & 4) << 4 | (v & 8) << 6; }
 
 __global__ void __launch_bounds__(PC_WG) k_nn_box(NnPair a) {
@@ -125,13 +129,19 @@ __global__ void __launch_bounds__(PC_WG) k_nn_box(NnPair a) {
     NnCloud c = a.c[blockIdx.y];
     for (int k = blockIdx.x * PC_WG + threadIdx.x; k < NN_CELLS; k += NN_BOXES * PC_WG) c.count[k] = 0;
     float v[6] = {INFINITY, INFINITY, INFINITY, INFINITY, INFINITY, INFINITY};
-    for (int i = blockIdx.x * PC_WG + threadIdx.x; i < c.n; i += NN_BOXES * PC_WG)
+    // every NN_BOXES'th run of 8 points: each partial box is a sample of the whole cloud
+    int per = PC_WG / 8;
+    for (long long r = blockIdx.x + (long long)(threadIdx.x >> 3) * NN_BOXES; r * 8 < c.n; r += (long long)per * NN_BOXES) {
+        long long i = r * 8 + (threadIdx.x & 7);
+        if (i >= c.n) continue;
+        float u[3] = {c.p[i * 3], c.p[i * 3 + 1], c.p[i * 3 + 2]};
+        if (nn_special(u[0], u[1], u[2])) continue;
 #pragma unroll
         for (int d = 0; d < 3; d++) {
-            float u = c.p[(size_t)i * 3 + d];
-            v[d] = fminf(v[d], u);
-            v[3 + d] = fminf(v[3 + d], -u);
+            v[d] = fminf(v[d], u[d]);
+            v[3 + d] = fminf(v[3 + d], -u[d]);
         }
+    }
 #pragma unroll
     for (int d = 0; d < 6; d++) {
         for (int o = 32; o > 0; o >>= 1) v[d] = fminf(v[d], __shfl_xor(v[d], o));
@@ -145,7 +155,12 @@ __global__ void __launch_bounds__(PC_WG) k_nn_box(NnPair a) {
     }
 }
 
-// each point's cell, and its rank in it
+// Each point's cell, and its rank in it.  The extent of an axis: of 16 samples (4
+// partial boxes each) the innermost ends, so that points which some sample does not
+// hold do not stretch it (with one outlier at 500 times the extent every other point
+// fell into one cell: 30000 x 25001 points one way 192 us, every pair 160).  The
+// others, by a few percent at the ends, go to the border cells; the blocks' boxes are
+// the points' own.
 __global__ void __launch_bounds__(PC_WG) k_nn_count(NnPair a) {
     NnCloud c = a.c[blockIdx.y];
     if ((int)blockIdx.x * PC_WG >= c.n) return;
@@ -154,9 +169,15 @@ __global__ void __launch_bounds__(PC_WG) k_nn_count(NnPair a) {
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         float mn = c.part[lane * 6 + d], mx = c.part[lane * 6 + 3 + d];
-        for (int o = 32; o > 0; o >>= 1) {
+        for (int o = 1; o < 4; o <<= 1) {
             mn = fminf(mn, __shfl_xor(mn, o));
             mx = fminf(mx, __shfl_xor(mx, o));
+        }
+        mn = mn < INFINITY ? mn : -INFINITY;   // (an empty sample)
+        mx = mx < INFINITY ? mx : -INFINITY;
+        for (int o = 4; o < 64; o <<= 1) {
+            mn = fmaxf(mn, __shfl_xor(mn, o));
+            mx = fmaxf(mx, __shfl_xor(mx, o));
         }
         lo[d] = mn;
         float w = -mx - mn;
@@ -167,7 +188,7 @@ __global__ void __launch_bounds__(PC_WG) k_nn_count(NnPair a) {
     int cell = 0;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        // (a NaN or infinity, in the point or in the box, ends in a border cell)
+        // (points outside the extent, at infinity or NaN end in a border cell)
         float u = (c.p[(size_t)i * 3 + d] - lo[d]) * scale[d];
         int k = (int)fminf(fmaxf(u, 0.f), (float)((1 << NN_BITS) - 1));
         cell |= nn_spread(k) << d;
@@ -211,14 +232,14 @@ __global__ void __launch_bounds__(1024) k_nn_sort(NnPair a) {
     }
 }
 
-// the blocks' boxes, half a wave each; padding and NaN do not count
+// the blocks' boxes, half a wave each; padding and special points do not count
 __global__ void __launch_bounds__(PC_WG) k_nn_blocks(NnPair a) {
     NnCloud c = a.c[blockIdx.y];
     int i = blockIdx.x * PC_WG + threadIdx.x;
     if ((int)blockIdx.x * PC_WG >= c.blocks * NN_BLOCK) return;
     bool in = i < c.blocks * NN_BLOCK;
     nn4 p = c.sorted[in ? i : 0];
-    bool real = in && __float_as_int(p.w) != 0x7fffffff;
+    bool real = in && __float_as_int(p.w) != 0x7fffffff && !nn_special(p.x, p.y, p.z);
     float v[6] = {real ? p.x : INFINITY, real ? p.y : INFINITY, real ? p.z : INFINITY,
                   real ? -p.x : INFINITY, real ? -p.y : INFINITY, real ? -p.z : INFINITY};
 #pragma unroll
@@ -269,11 +290,13 @@ __global__ void __launch_bounds__(NN_HALVES * NN_BLOCK) k_nn_search(NnPair a, in
     if ((int)blockIdx.x >= q.blocks) return;
     int tid = threadIdx.x, half = tid >> 5, ql = tid & 31;
     nn4 me = q.sorted[(size_t)blockIdx.x * NN_BLOCK + ql];
-    bool live = __float_as_int(me.w) != 0x7fffffff;
+    bool real = __float_as_int(me.w) != 0x7fffffff, live = real && !nn_special(me.x, me.y, me.z);
+    if (!live) me.x = me.y = me.z = INFINITY;
     nn4 lo = q.box[2 * (size_t)blockIdx.x], hi = q.box[2 * (size_t)blockIdx.x + 1];
     if (half == 0) {
         query[ql] = me;
-        // (a lane without a query neither asks for anything nor takes anything)
+        // (a lane without a query, or with one at no finite distance from any target,
+        // neither asks for anything nor takes anything)
         best[ql] = live ? nn_key(INFINITY, 0x7fffffff) : 0ull;
     }
     if (tid < 2) listed[tid] = 0;
@@ -343,11 +366,11 @@ __global__ void __launch_bounds__(NN_HALVES * NN_BLOCK) k_nn_search(NnPair a, in
         if (tid < 2) listed[tid] = 0;
     }
     __syncthreads();
-    if (half != 0 || !live) return;
+    if (half != 0 || !real) return;
     unsigned long long k = best[ql];
     float bd = __uint_as_float((unsigned)(k >> 32));
     int at = __float_as_int(me.w);
-    bool nothing = !(bd < INFINITY);
+    bool nothing = !live || !(bd < INFINITY);
     (dir ? idx1 : idx0)[at] = nothing ? -1 : (int)(unsigned)k;
     (dir ? d1 : d0)[at] = nothing ? INFINITY : bd;
 }
