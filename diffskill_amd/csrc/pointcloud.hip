@@ -981,14 +981,24 @@ int sk_splits(int n, int m) {
     return std::max(1, std::min(s, 65535));
 }
 
-// whether the search over every pair takes a direction with nt targets: when it
-// is wanted alone and they are few (us, one direction of 250 x 250 points: 19.0
-// against 24.5 sorted, 500 x 500: 23.6 against 24.5, 1000 x 1000: 41.6 against
-// 24.4; both ways at 250: 30.5 against 27.1), or as the only one that can (no
-// targets, more than it takes)
+// Which search takes a call: the times of both, us, as measured over 1 to 1000000
+// points on either side.  Every pair: a workgroup passes over up to 2048 targets,
+// 6.0e6 pairs a us once the chip is full.  Sorted: five launches, a term for each
+// cloud's sort (targets more than queries: few queries leave few workgroups to
+// go over many blocks' boxes) and one for the blocks' boxes, a pair of blocks each.
+// One way, queries x targets, every pair against sorted: 300 x 300 15.4, 16.7;
+// 300 x 1000 39.9, 20.5; 40000 x 600 27.9, 31.3; 40000 x 1000 42.9, 34.4; 1000 x
+// 40000 83, 69; 300 x 100000 83, 118; 10000 x 100000 198, 84; 100 x 1000000 85, 792;
+// 1000000 x 1000 187, 419; 1000000 x 4000 650, 521; 200000 x 150000 4566, 326.  Both
+// ways: 300 x 100 25, 16.3; 200000 x 600 127, 181; 200000 x 4000 350, 199; 100 x
+// 1000000 115, 808.
+double nn_every_us(double nq, double nt) { return std::max(5.0 + 0.0375 * std::min(nt, (double)PC_CHUNK), nq * nt / 6.0e6); }
+// (also without targets, or with more than the sorted search takes)
 bool nn_brute(int n, int m, bool do_x, bool do_y) {
     if (n == 0 || m == 0 || n > 65535 * PC_CHUNK || m > 65535 * PC_CHUNK) return true;
-    return do_x != do_y && (do_x ? m : n) <= 512;
+    if (do_x && do_y) return nn_every_us(n, m) + nn_every_us(m, n) <= 16.5 + 0.8e-3 * ((double)n + m) + (double)n * m / 1.0e8;
+    double nq = do_x ? n : m, nt = do_x ? m : n;
+    return nn_every_us(nq, nt) <= 16.5 + 0.4e-3 * nq + 0.7e-3 * nt + nq * nt / 2.0e8;
 }
 
 }  // namespace
