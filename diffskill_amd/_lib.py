@@ -53,7 +53,7 @@ EXPORTS = [
     "mpm_resort_bytes", "mpm_set_resort", "mpm_get_resort", "mpm_slot_order",
     "pc_nearest", "pc_nearest_noalloc", "pc_last_error", "pc_sinkhorn_work_bytes", "pc_softmin", "pc_plan_grad",
     "pc_sinkhorn_step_work_bytes", "pc_sinkhorn_step", "pc_sinkhorn_solve", "pc_sinkhorn_grad", "pc_extent",
-    "pc_nearest_pair_work_bytes", "pc_nearest_pair", "pc_chamfer_loss", "pc_chamfer_grad",
+    "pc_nearest_pair_work_bytes", "pc_nearest_pair", "pc_chamfer_loss", "pc_chamfer", "pc_chamfer_grad",
 ]
 
 PHASES = ["bin", "compact", "blocks", "scatter", "stress", "p2g", "grid_op", "g2p", "p2g_grid", "grid_op_keep",
@@ -132,6 +132,7 @@ def load():
         "pc_nearest_pair_work_bytes": (ctypes.c_longlong, [i32, i32]),
         "pc_nearest_pair": (i32, [vp, i32, vp, i32, vp, vp, vp, vp, vp, vp]),
         "pc_chamfer_loss": (i32, [vp, i32, vp, i32, i32, vp, vp]),
+        "pc_chamfer": (i32, [vp, i32, vp, i32, i32, vp, vp, vp, vp, vp, vp, vp]),
         "pc_chamfer_grad": (i32, [vp, i32, vp, i32, vp, vp, vp, vp, i32, vp, vp, vp, vp]),
         "pc_last_error": (ctypes.c_char_p, []),
     }

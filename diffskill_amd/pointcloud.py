@@ -151,38 +151,45 @@ class _Chamfer(torch.autograd.Function):
     def forward(ctx, x, y, bidirectional, squared):
         L = _lib.load()
         xd, yd = _cloud(x, "q"), _cloud(y, "t")
-        px, py = _nearest_pair(xd, yd, (True, bidirectional))
-        ix, dx = px
-        iy, dy = py if bidirectional else (None, None)
+        n, m = xd.shape[0], yd.shape[0]
+        # int32 indices, then squared distances, of x's points; the same of y's
+        near = torch.empty(2 * (n + m) if bidirectional else 2 * n, dtype=torch.float32, device=xd.device)
         loss = torch.empty((), dtype=torch.float32, device=xd.device)
-        _check("pc_chamfer_loss", L.pc_chamfer_loss(_p(dx), xd.shape[0], _p(dy) if bidirectional else None, yd.shape[0], int(squared),
-                                                    _p(loss), _stream()))
-        ctx.save_for_backward(x, y, ix, dx, iy, dy)
-        ctx.squared = squared
+        work = torch.empty((L.pc_nearest_pair_work_bytes(n, m) + 15) // 16 * 4, dtype=torch.float32, device=xd.device)
+        _check("pc_chamfer", L.pc_chamfer(xd.data_ptr(), n, yd.data_ptr(), m, squared, work.data_ptr(),
+                                          *_Chamfer.ptrs(near, n, m, bidirectional), loss.data_ptr(), _stream()))
+        ctx.save_for_backward(x, y, near)
+        ctx.bidirectional, ctx.squared = bidirectional, squared
         return loss
 
     @staticmethod
+    def ptrs(near, n, m, both):
+        at = near.data_ptr()
+        return (at, at + 4 * n) + ((at + 8 * n, at + 8 * n + 4 * m) if both else (None, None))
+
+    @staticmethod
     def backward(ctx, go):
-        x, y, ix, dx, iy, dy = ctx.saved_tensors
-        want = ctx.needs_input_grad
+        x, y, near = ctx.saved_tensors
+        want_x, want_y = ctx.needs_input_grad[:2]
         n, m = x.shape[0], y.shape[0]
         if torch.is_grad_enabled() or not _has_memory(go) or torch.are_deterministic_algorithms_enabled():
             # a gradient that is to be differentiated again, a batch of them, or one
             # summed in a fixed order (pc_chamfer_grad's sums over the points that
             # share a target have none): in operations that take those
-            def one(p, t, idx, d2, w):
-                return _distance_grad(p, t, idx.long(), d2 if ctx.squared else torch.sqrt(d2), ctx.squared,
-                                      (go / p.shape[0]).expand(p.shape[0]), w)
-            gx, gy = one(x, y, ix, dx, want[1])
-            if iy is not None:
-                hy, hx = one(y, x, iy, dy, want[0])
-                gx, gy = (gx + hx if want[0] else None), (gy + hy if want[1] else None)
-            return gx if want[0] else None, gy, None, None
-        xd, yd = _cloud(x, "q"), _cloud(y, "t")
-        gx, gy = (torch.empty_like(c) if w else None for c, w in zip((xd, yd), want))
+            def one(p, t, at, w):
+                k = len(p)
+                idx, d2 = near[at:at + k].view(torch.int32).long(), near[at + k:at + 2 * k]
+                return _distance_grad(p, t, idx, d2 if ctx.squared else torch.sqrt(d2), ctx.squared, (go / k).expand(k), w)
+            gx, gy = one(x, y, 0, want_y)
+            if ctx.bidirectional:
+                hy, hx = one(y, x, 2 * n, want_x)
+                gx, gy = (gx + hx if want_x else None), (gy + hy if want_y else None)
+            return gx if want_x else None, gy, None, None
+        xd, yd = x.contiguous(), y.contiguous()
+        gx, gy = (torch.empty_like(c) if w else None for c, w in ((xd, want_x), (yd, want_y)))
         _check("pc_chamfer_grad", _lib.load().pc_chamfer_grad(
-            _p(xd), n, _p(yd), m, _p(ix), _p(dx), None if iy is None else _p(iy), None if dy is None else _p(dy), int(ctx.squared),
-            _p(go.contiguous()), None if gx is None else _p(gx), None if gy is None else _p(gy), _stream()))
+            xd.data_ptr(), n, yd.data_ptr(), m, *_Chamfer.ptrs(near, n, m, ctx.bidirectional), ctx.squared, go.data_ptr(),
+            gx.data_ptr() if want_x else None, gy.data_ptr() if want_y else None, _stream()))
         return gx, gy, None, None
 
 

@@ -129,6 +129,12 @@ int pc_nearest_pair(const float *x, int n, const float *y, int m, void *work, in
  * squares with squared != 0.  One launch. */
 int pc_chamfer_loss(const float *d2_x, int n, const float *d2_y, int m, int squared, float *out, void *stream);
 
+/* Search and loss in one call: pc_nearest_pair into idx_x, d2_x and, unless null,
+ * idx_y, d2_y, and the loss of these directions to loss[0].  Both clouds non-empty;
+ * work as for pc_nearest_pair. */
+int pc_chamfer(const float *x, int n, const float *y, int m, int squared, void *work, int *idx_x, float *d2_x, int *idx_y, float *d2_y,
+               float *loss, void *stream);
+
 /* Its gradient times *go (device float) in both clouds, the indices held:
  * gx (n x 3) and gy (m x 3) are overwritten, either may be null; idx_y and d2_y
  * null for a loss of x's direction alone.  A point without a nearest target gets

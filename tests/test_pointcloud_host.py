@@ -62,13 +62,13 @@ def _zeros(p, nbytes):
     return 0
 
 
-def _search(x, n, y, m, work, ix, dx, iy, dy, stream):
+def _search(x, n, y, m, squared, work, ix, dx, iy, dy, loss, stream):
     """Every point's nearest target is target 0, at distance 0."""
     return _zeros(ix, 4 * n) or _zeros(dx, 4 * n) or _zeros(iy, 4 * m) or _zeros(dy, 4 * m)
 
 
 def _chamfer_library():
-    return Library(pc_nearest_pair_work_bytes=64, pc_nearest_pair=_search)
+    return Library(pc_nearest_pair_work_bytes=64, pc_chamfer=_search)
 
 
 @pytest.mark.parametrize("both", [False, True])
