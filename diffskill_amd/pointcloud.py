@@ -43,7 +43,9 @@ from . import _lib
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # (torch.cuda.current_stream() takes 16 us in a loss's forward and backward
+    # passes, this 3; their library calls take 19 and 10)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _p(t):
