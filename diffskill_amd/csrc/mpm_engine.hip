@@ -3,9 +3,10 @@
 // One context packs any number of scenes (each with its own grid and tool
 // primitives) into shared device arrays, so every phase of a substep is ONE
 // launch over all scenes:
-//   forward  : mark(+primitive FK) -> compact -> p2g -> grid_op -> g2p
-//   adjoint  : mark -> compact -> p2g -> grid_op(keep) -> g2p_bwd ->
-//              grid_op_bwd -> p2g_bwd(+primitive FK adjoint)
+//   forward  : bin (+ primitive FK) -> blocks (+ constitutive update) ->
+//              scatter -> p2g -> grid_op -> g2p (+ the next frame's bin)
+//   adjoint  : g2p_bwd -> grid_op_bwd -> p2g_bwd (+ constitutive adjoint,
+//              primitive FK adjoint), over the forward's kept lists and grid
 // The reference runs the same sequence as ~7 + n_prim Taichi launches per
 // scene and substep (plb/engine/mpm_simulator.py:307-345).
 //

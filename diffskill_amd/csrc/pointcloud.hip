@@ -1,14 +1,15 @@
-// Point-cloud nearest neighbours on gfx950: the search under the Chamfer
-// losses of the reference (plb/engine/losses/loss.py:183-204, and the
-// chamferdist.ChamferDistance loss of plb/engine/taichi_env.py:28-32).
+// Point-cloud losses on gfx950: the nearest-neighbour searches under the
+// Chamfer losses of the reference (plb/engine/losses/loss.py:183-204, and the
+// chamferdist.ChamferDistance loss of plb/engine/taichi_env.py:28-32), those
+// losses and their gradients, and the Sinkhorn divergence of its EMD loss.
 //
-// Brute force over all (query, target) pairs, exact in fp32: a workgroup
-// takes 256 queries (one per lane) and one chunk of targets staged in LDS;
-// every lane scans the chunk (LDS broadcast reads) keeping its smallest
-// squared distance and the first index reaching it.  Chunks meet through one
-// 64-bit atomicMin per query on (distance bits << 32 | index): distances are
-// non-negative, so their bit patterns order like the values, and equal
-// distances keep the smaller index.
+// Nearest neighbours, every pair: brute force over all (query, target) pairs,
+// exact in fp32: a workgroup takes 256 queries (one per lane) and one chunk of
+// targets staged in LDS; every lane scans the chunk (LDS broadcast reads)
+// keeping its smallest squared distance and the first index reaching it.
+// Chunks meet through one 64-bit atomicMin per query on (distance bits << 32 |
+// index): distances are non-negative, so their bit patterns order like the
+// values, and equal distances keep the smaller index.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>
@@ -99,7 +100,7 @@ __global__ void __launch_bounds__(PC_WG) k_pc_nearest(const float* __restrict__ 
 // a comparison that NaN or infinities spoil scans.
 // What bounds it: five dependent launches (about 4 us each) and, in the search, the
 // latency of the block loads.  Both ways, every pair -> sorted: 30000 x 25001
-// points 309 -> 64 us, 10000 x 10000 166 -> 35, 3000 x 3000 164 -> 28 (the search
+// points 309 -> 67 us, 10000 x 10000 166 -> 36, 3000 x 3000 164 -> 24 (the search
 // over every pair gives a workgroup 2048 targets at least).
 constexpr int NN_BITS = 4, NN_CELLS = 1 << (3 * NN_BITS);
 constexpr int NN_BLOCK = 32;
@@ -376,10 +377,11 @@ __global__ void __launch_bounds__(NN_HALVES * NN_BLOCK) k_nn_search(NnPair a, in
 }
 
 // ------------------------------------------------- Chamfer loss and gradient
-// From pc_nearest_pair's outputs: the loss (fp64 sums in a fixed order), the gradient in two launches -- every point's own term stored, then
-// the terms of the points that chose it added -- where the elementwise
-// operations of a framework took about 40 (30000 x 25001 points both ways, forward
-// and gradients after the search: 130 -> 34 us of kernels).
+// From pc_nearest_pair's outputs: the loss (fp64 sums in a fixed order) in one launch
+// or two, the gradient in two -- every point's own term stored, then the terms of
+// the points that chose it added -- or three, where the elementwise operations of
+// a framework took about 40 (30000 x 25001 points both ways, forward and gradients
+// after the search: 130 -> 18 us of kernels).
 struct ChDir { const float* p; const float* t; const int* idx; const float* d2; float* gp; float* gt; int n; };
 
 // one workgroup: the loss; several: their sums to part[direction][workgroup], which

@@ -13,7 +13,10 @@ import torch
 
 
 def default_candidates(n_cu):
-    """(particles_per_item, tile_ctas, grid_ctas) shapes to try."""
+    """(particles_per_item, tile_ctas, grid_ctas) shapes to try.  (Items of 2048
+    were 2 to 20 % slower than the best in contexts of 200 thousand to 1.6 million
+    particles, 1536 within 1 % of it at most: 64 scenes 257 us a forward and adjoint
+    substep at 768, 271 at 2048; 16 of 100000 417, 428; one of 1200000 356, 364.)"""
     return [(ppi, t * n_cu, 8 * n_cu) for ppi in (256, 512, 768, 1024) for t in (2, 4, 8)]
 
 

@@ -117,8 +117,8 @@ int pc_extent(const float *x, int n, const float *y, int m, float *out, void *st
  * of x (idx_y, d2_y); a direction whose two outputs are null is left out.
  * Indices and squared distances are pc_nearest's, bit for bit, an empty target
  * cloud's included.  work: pc_nearest_pair_work_bytes(n, m) device bytes, 16-byte
- * aligned.  Clouds of more than a few hundred points are sorted spatially and most
- * pairs are left out.  Asynchronous on stream, no allocation.  Returns 0, or
+ * aligned.  Either every pair is looked at, or both clouds are sorted spatially and
+ * most pairs left out, whichever is the faster at these sizes.  Asynchronous on stream, no allocation.  Returns 0, or
  * -1 with pc_last_error(). */
 long long pc_nearest_pair_work_bytes(int n, int m);
 int pc_nearest_pair(const float *x, int n, const float *y, int m, void *work, int *idx_x, float *d2_x, int *idx_y, float *d2_y,
@@ -138,7 +138,7 @@ int pc_chamfer(const float *x, int n, const float *y, int m, int squared, void *
 /* Its gradient times *go (device float) in both clouds, the indices held:
  * gx (n x 3) and gy (m x 3) are overwritten, either may be null; idx_y and d2_y
  * null for a loss of x's direction alone.  A point without a nearest target gets
- * NaN.  Two launches; sums over the points that share a target are atomic, in no
+ * NaN.  Two or three launches; sums over the points that share a target are atomic, in no
  * fixed order. */
 int pc_chamfer_grad(const float *x, int n, const float *y, int m, const int *idx_x, const float *d2_x, const int *idx_y,
                     const float *d2_y, int squared, const float *go, float *gx, float *gy, void *stream);
