@@ -48,7 +48,7 @@ ALGO_BYTES = {
 
 
 # engine phase -> kernel name in the rocprof summaries
-PHASE_KERNEL = {"stress": "k_stress", "p2g": "k_p2g_scatter", "p2g_grid": "k_p2g_scatter_rebuild", "g2p": "k_g2p",
+PHASE_KERNEL = {"stress": "k_stress", "p2g": "k_p2g_scatter", "p2g_grid": "k_p2g_scatter_rebuild", "g2p": "k_g2p<false>",
                 "g2p_bwd": "k_g2p_bwd_tile", "p2g_bwd": "k_p2g_bwd", "bin": "k_bin",
                 "grid_op": "k_grid_op", "grid_op_keep": "k_grid_op_rebuild", "grid_op_bwd": "k_grid_op_bwd"}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_batched64_config4.json")
