@@ -104,7 +104,8 @@ __global__ void __launch_bounds__(PC_WG) k_pc_nearest(const float* __restrict__ 
 // over every pair gives a workgroup 2048 targets at least).
 constexpr int NN_BITS = 4, NN_CELLS = 1 << (3 * NN_BITS);
 constexpr int NN_BLOCK = 32;
-constexpr int NN_BOXES = 64;       // workgroups, and partial boxes, of k_nn_box
+constexpr int NN_RUNS = 1 << 16;    // points from which k_nn_box reads runs
+constexpr int NN_BOXES = 61;       // workgroups, and partial boxes, of k_nn_box: a wave's lanes at most, and prime
 constexpr int NN_LIST = 1024;      // target blocks tested at a time
 constexpr float NN_MARGIN = 0.999999f;
 typedef float nn4 __attribute__((ext_vector_type(4)));
@@ -130,10 +131,13 @@ __global__ void __launch_bounds__(PC_WG) k_nn_box(NnPair a) {
     NnCloud c = a.c[blockIdx.y];
     for (int k = blockIdx.x * PC_WG + threadIdx.x; k < NN_CELLS; k += NN_BOXES * PC_WG) c.count[k] = 0;
     float v[6] = {INFINITY, INFINITY, INFINITY, INFINITY, INFINITY, INFINITY};
-    // every NN_BOXES'th run of 8 points: each partial box is a sample of the whole cloud
-    int per = PC_WG / 8;
-    for (long long r = blockIdx.x + (long long)(threadIdx.x >> 3) * NN_BOXES; r * 8 < c.n; r += (long long)per * NN_BOXES) {
-        long long i = r * 8 + (threadIdx.x & 7);
+    // every NN_BOXES'th point, or run of 8 in large clouds: each partial box is a sample
+    // of the whole cloud (a prime number of them, so that the rows of a lattice, 16, 32
+    // or 64 points long, do not give each sample a stretch of its own of the axis they
+    // run along; points by themselves while there are few runs to a sample)
+    int run = c.n > NN_RUNS ? 3 : 0, per = PC_WG >> run;
+    for (long long r = blockIdx.x + (long long)(threadIdx.x >> run) * NN_BOXES; r << run < c.n; r += (long long)per * NN_BOXES) {
+        long long i = (r << run) + (threadIdx.x & ((1 << run) - 1));
         if (i >= c.n) continue;
         float u[3] = {c.p[i * 3], c.p[i * 3 + 1], c.p[i * 3 + 2]};
         if (nn_special(u[0], u[1], u[2])) continue;
@@ -169,7 +173,7 @@ __global__ void __launch_bounds__(PC_WG) k_nn_count(NnPair a) {
     float lo[3], scale[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        float mn = c.part[lane * 6 + d], mx = c.part[lane * 6 + 3 + d];
+        float mn = lane < NN_BOXES ? c.part[lane * 6 + d] : INFINITY, mx = lane < NN_BOXES ? c.part[lane * 6 + 3 + d] : INFINITY;
         for (int o = 1; o < 4; o <<= 1) {
             mn = fminf(mn, __shfl_xor(mn, o));
             mx = fminf(mx, __shfl_xor(mx, o));

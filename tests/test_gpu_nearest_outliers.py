@@ -18,6 +18,9 @@ def _cloud(n, kind, seed):
     x = torch.rand((n, 3), generator=g)
     if kind == "ordered":          # along an axis, as a lattice or a scan comes
         x = x[x[:, 0].argsort()]
+    elif kind == "lattice":        # rows of 64 points along one axis
+        k = torch.arange(n)
+        x = torch.stack([k // 64 // 16, k // 64 % 16, k % 64], 1) / 64.0 + 0.001 * x
     elif kind == "one":
         x[n // 2] = 500.0 * (1 if seed % 2 else -1)
     elif kind == "few":
@@ -33,7 +36,7 @@ def _cloud(n, kind, seed):
 
 
 @pytest.mark.parametrize("n,m", [(6, 9), (40, 31), (700, 600), (3000, 2999), (20000, 5001)])
-@pytest.mark.parametrize("kind", ["ordered", "one", "few", "huge", "infinite", "special"])
+@pytest.mark.parametrize("kind", ["ordered", "lattice", "one", "few", "huge", "infinite", "special"])
 def test_outliers(n, m, kind):
     from diffskill_amd import _lib
     L = _lib.load()
@@ -53,4 +56,5 @@ def test_outliers(n, m, kind):
         # a few of which take 3000 or more points' outliers
         at = (n + 31) // 32 * (32 * 16 + 32)
         cells = work[at:at + 8 * n].view(torch.int32)[::2]
-        assert 1500 < len(cells.unique()) <= 4096
+        rows = -(-n // (64 * 16)) if kind == "lattice" else 16
+        assert 1500 * min(16, rows) // 16 < len(cells.unique()) <= 4096
