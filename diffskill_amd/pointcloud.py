@@ -97,15 +97,21 @@ def _nearest_pair(x, y, want):
     return out
 
 
-def _distance_grad(x, y, idx, d, squared, g, want_y):
-    """Gradients in x and y of d_i = |x_i - y_idx(i)| (or its square) times g."""
+def _distance_grad(x, y, idx, d, squared, g, want_y, none=None):
+    """Gradients in x and y of d_i = |x_i - y_idx(i)| (or its square) times g; NaN
+    for the points of x in ``none``, which have no nearest y."""
+    if none is not None:
+        idx = idx.clamp_min(0)
     diff = x - y.index_select(0, idx)
+    if none is not None:
+        diff = diff.masked_fill(none[:, None], 0.0)
     if squared:
         gx = 2.0 * diff * g[:, None]
     else:
         inv = torch.where(d > 0, 1.0 / d.clamp_min(1e-30), torch.zeros_like(d))
         gx = diff * (g * inv.to(g.dtype))[:, None]
-    return gx, torch.zeros_like(y).index_add(0, idx, -gx) if want_y else None
+    gy = torch.zeros_like(y).index_add(0, idx, -gx) if want_y else None
+    return gx if none is None else gx.masked_fill(none[:, None], float("nan")), gy
 
 
 class _NearestDistance(torch.autograd.Function):
@@ -181,7 +187,7 @@ class _Chamfer(torch.autograd.Function):
             def one(p, t, at, w):
                 k = len(p)
                 idx, d2 = near[at:at + k].view(torch.int32).long(), near[at + k:at + 2 * k]
-                return _distance_grad(p, t, idx, d2 if ctx.squared else torch.sqrt(d2), ctx.squared, (go / k).expand(k), w)
+                return _distance_grad(p, t, idx, d2 if ctx.squared else torch.sqrt(d2), ctx.squared, (go / k).expand(k), w, idx < 0)
             gx, gy = one(x, y, 0, want_y)
             if ctx.bidirectional:
                 hy, hx = one(y, x, 2 * n, want_x)

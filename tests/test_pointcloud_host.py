@@ -117,3 +117,25 @@ def test_chamfer_gradient_of_deterministic_algorithms(host, fixed):
     assert ("pc_chamfer_grad" in lib.seen) != fixed
     if fixed:
         assert torch.allclose(gx, 2 * (x - y[0]) / 5) and torch.allclose(gy[0], -gx.sum(0)) and (gy[1:] == 0).all()
+
+
+@pytest.mark.parametrize("squared", [False, True])
+def test_chamfer_gradient_without_a_nearest_target(host, squared):
+    """A point at infinity: NaN for itself, nothing for the targets, in torch's
+    operations as in the kernel (where an index of -1 stopped the program)."""
+    def search(x, n, y, m, squared, work, ix, dx, iy, dy, loss, stream):
+        idx = (ctypes.c_int * n)(*[-1 if k == 2 else 0 for k in range(n)])
+        d2 = (ctypes.c_float * n)(*[float("inf") if k == 2 else 4.0 for k in range(n)])
+        ctypes.memmove(ix, idx, 4 * n)
+        ctypes.memmove(dx, d2, 4 * n)
+        return 0
+
+    host(Library(pc_nearest_pair_work_bytes=64, pc_chamfer=search))
+    x, y = torch.rand(5, 3), torch.rand(4, 3, requires_grad=True)
+    x[2] = float("inf")
+    x.requires_grad_(True)
+    gx, gy = torch.autograd.grad(pc.chamfer_distance(x, y, squared=squared), (x, y), create_graph=True)
+    keep = [0, 1, 3, 4]
+    ref = ((2.0 if squared else 0.5) * (x - y[0]) / 5)[keep]
+    assert torch.isnan(gx[2]).all() and torch.allclose(gx[keep], ref)
+    assert torch.allclose(gy[0], -ref.sum(0)) and (gy[1:] == 0).all()
