@@ -160,8 +160,9 @@ class _Chamfer(torch.autograd.Function):
         L = _lib.load()
         xd, yd = _cloud(x, "q"), _cloud(y, "t")
         n, m = xd.shape[0], yd.shape[0]
-        # int32 indices, then squared distances, of x's points; the same of y's
-        near = torch.empty(2 * (n + m) if bidirectional else 2 * n, dtype=torch.float32, device=xd.device)
+        # indices, then squared distances (their bits), of x's points; the same of y's.
+        # (integers: what a saved-tensor hook may do to floats would be other indices)
+        near = torch.empty(2 * (n + m) if bidirectional else 2 * n, dtype=torch.int32, device=xd.device)
         loss = torch.empty((), dtype=torch.float32, device=xd.device)
         work = torch.empty((L.pc_nearest_pair_work_bytes(n, m) + 15) // 16 * 4, dtype=torch.float32, device=xd.device)
         _check("pc_chamfer", L.pc_chamfer(xd.data_ptr(), n, yd.data_ptr(), m, squared, work.data_ptr(),
@@ -186,14 +187,16 @@ class _Chamfer(torch.autograd.Function):
             # share a target have none): in operations that take those
             def one(p, t, at, w):
                 k = len(p)
-                idx, d2 = near[at:at + k].view(torch.int32).long(), near[at + k:at + 2 * k]
+                idx, d2 = near[at:at + k].long(), near[at + k:at + 2 * k].view(torch.float32)
                 return _distance_grad(p, t, idx, d2 if ctx.squared else torch.sqrt(d2), ctx.squared, (go / k).expand(k), w, idx < 0)
             gx, gy = one(x, y, 0, want_y)
             if ctx.bidirectional:
                 hy, hx = one(y, x, 2 * n, want_x)
                 gx, gy = (gx + hx if want_x else None), (gy + hy if want_y else None)
             return gx if want_x else None, gy, None, None
-        xd, yd = x.contiguous(), y.contiguous()
+        # (as the kernel reads them, whatever came back from the hooks)
+        xd, yd = _cloud(x, "q"), _cloud(y, "t")
+        near = near.to(xd.device, torch.int32).contiguous()
         gx, gy = (torch.empty_like(c) if w else None for c, w in ((xd, want_x), (yd, want_y)))
         _check("pc_chamfer_grad", _lib.load().pc_chamfer_grad(
             xd.data_ptr(), n, yd.data_ptr(), m, *_Chamfer.ptrs(near, n, m, ctx.bidirectional), ctx.squared, go.data_ptr(),

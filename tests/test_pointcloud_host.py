@@ -139,3 +139,27 @@ def test_chamfer_gradient_without_a_nearest_target(host, squared):
     ref = ((2.0 if squared else 0.5) * (x - y[0]) / 5)[keep]
     assert torch.isnan(gx[2]).all() and torch.allclose(gx[keep], ref)
     assert torch.allclose(gy[0], -ref.sum(0)) and (gy[1:] == 0).all()
+
+
+def test_chamfer_saved_tensor_hooks(host):
+    """Hooks that keep floats at half precision: the gradient kernel still gets
+    float32 clouds and the search's own indices."""
+    seen = {}
+
+    def search(x, n, y, m, squared, work, ix, dx, iy, dy, loss, stream):
+        ctypes.memmove(ix, (ctypes.c_int * n)(*range(100000, 100000 + n)), 4 * n)
+        return _zeros(dx, 4 * n)
+
+    def grad(x, n, y, m, ix, dx, iy, dy, squared, go, gx, gy, stream):
+        seen["idx"] = list((ctypes.c_int * n).from_address(ix))
+        seen["x"] = list((ctypes.c_float * (3 * n)).from_address(x))
+        return _zeros(gx, 12 * n) or _zeros(gy, 12 * m)
+
+    host(Library(pc_nearest_pair_work_bytes=64, pc_chamfer=search, pc_chamfer_grad=grad))
+    x, y = torch.rand(5, 3, requires_grad=True), torch.rand(4, 3, requires_grad=True)
+    half = lambda t: t.half() if t.is_floating_point() else t   # noqa: E731
+    with torch.autograd.graph.saved_tensors_hooks(half, lambda t: t):
+        loss = pc.chamfer_distance(x, y)
+    loss.backward()
+    assert seen["idx"] == list(range(100000, 100005))
+    assert seen["x"] == x.detach().half().float().flatten().tolist()
